@@ -15,6 +15,7 @@ import numpy as np
 import pytest
 
 import mnb_hip
+import mnb_oracle as orc
 from mnb_hip import synth
 
 pytestmark = pytest.mark.gpu
@@ -184,3 +185,59 @@ def test_graph_capture_of_tile_list_groups():
     finally:
         torch.cuda.synchronize()
         ctx.close()
+
+
+@pytest.mark.parametrize("mode,other_thread", [("relaxed", False), ("relaxed", True), ("thread_local", True)])
+def test_quantized_weight_destroyed_during_a_capture(mode, other_thread):
+    """A quantized weight is destroyed while a stream is being captured, by the
+    capturing thread or another one, in the capture modes that allow a
+    hipFree: the weight closes, the capture goes on and its replays equal the
+    eager products, and a weight quantized next equals the reference's."""
+    import threading
+    import torch
+    ctx = mnb_hip.Context(0)
+    rng = np.random.default_rng(8)
+    N, K = 896, 896
+    t = synth.make_weight(8, N, K, 32)
+    w = mnb_hip.Weight(ctx, N, K, 32, t.q, t.scales_f16)
+    table = (0.05 * rng.standard_normal((2048, K))).astype(np.float32)
+    gone = mnb_hip.Weight.quantize(ctx, table)
+    x = torch.randn((1, K), device="cuda").half()
+    y, y2, ref = (torch.empty((1, N), device="cuda") for _ in range(3))
+    torch.cuda.synchronize()
+    errors = []
+
+    def close():
+        try:
+            gone.close()
+        except Exception as e:  # noqa: BLE001  (a thread's exception would be lost)
+            errors.append(e)
+
+    st = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st, capture_error_mode=mode):
+        w.matmul(x, y, stream=st.cuda_stream)
+        if other_thread:
+            th = threading.Thread(target=close)
+            th.start()
+            th.join()
+        else:
+            close()
+        w.matmul(x, y2, stream=st.cuda_stream)
+    assert not errors, errors
+    for seed in range(3):
+        x.copy_(torch.randn((1, K), generator=torch.Generator("cuda").manual_seed(seed), device="cuda").half())
+        torch.cuda.synchronize()
+        w.matmul(x, ref, stream=st.cuda_stream)
+        with torch.cuda.stream(st):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, ref) and torch.equal(y2, ref)
+    nxt = mnb_hip.Weight.quantize(ctx, table[::-1].copy())
+    q, s, z = nxt.read()
+    rq, rs, rz = orc.quantize_rows_u4(table[::-1].copy(), 2048, K, 128)
+    assert np.array_equal(q, rq) and np.array_equal(s, rs) and np.array_equal(z, rz)
+    nxt.close()
+    w.close()
+    del graph
+    ctx.close()

@@ -98,20 +98,24 @@ hipError_t block_alloc(mnb_context *ctx, void **p, size_t bytes, size_t *got) {
 
 // Frees a weight's block, or keeps it as the context's spare one.  hipFree
 // waits for all work on the device, so a caller may destroy a weight whose
-// products are still running on any stream; a kept block is waited for the
-// same way.
-hipError_t block_free(mnb_context *ctx, void *block, size_t bytes) {
+// products are still running on any stream.  A kept block is waited for in
+// the same way, by freeing the weight's `fence`: hipDeviceSynchronize would
+// fail during a stream capture of any thread, and end that capture, where
+// hipFree is allowed (relaxed captures, other threads' thread-local ones).
+hipError_t block_free(mnb_context *ctx, void *block, size_t bytes, void *fence) {
     void *drop = block;
-    if (bytes <= mnb::kSpareMaxBytes) {
-        const hipError_t e = hipDeviceSynchronize();
+    if (fence) {
+        const hipError_t e = hipFree(fence);
         if (e != hipSuccess) {
             (void)hipFree(block);
             return e;
         }
-        std::lock_guard<std::mutex> lock(ctx->spare_mutex);
-        drop = ctx->spare;
-        ctx->spare = block;
-        ctx->spare_bytes = bytes;
+        if (bytes <= mnb::kSpareMaxBytes) {
+            std::lock_guard<std::mutex> lock(ctx->spare_mutex);
+            drop = ctx->spare;
+            ctx->spare = block;
+            ctx->spare_bytes = bytes;
+        }
     }
     return drop ? hipFree(drop) : hipSuccess;
 }
@@ -543,7 +547,8 @@ int32_t mnb_weight_quantize(mnb_context *ctx, const void *data, int32_t data_typ
     auto up = [](size_t v) { return (v + 255) & ~(size_t)255; };
     const size_t s_at = up(q_t_bytes), z_at = s_at + up(s_t_bytes), scratch_at = z_at + up(z_t_bytes);
     int32_t fold = 0;
-    if ((e = block_alloc(ctx, &w->q_t, scratch_at + mnb::kQuantScratchBytes, &w->block_bytes)) == hipSuccess) {
+    if ((e = block_alloc(ctx, &w->q_t, scratch_at + mnb::kQuantScratchBytes, &w->block_bytes)) == hipSuccess &&
+        (e = dev_alloc(ctx, &w->fence, 16)) == hipSuccess) {
         unsigned char *base = (unsigned char *)w->q_t;
         w->s_t = base + s_at;
         w->zp_t = base + z_at;
@@ -554,7 +559,7 @@ int32_t mnb_weight_quantize(mnb_context *ctx, const void *data, int32_t data_typ
     }
     if (staged) (void)hipFree(staged);
     if (e != hipSuccess) {
-        if (w->q_t) (void)block_free(ctx, w->q_t, w->block_bytes);
+        if (w->q_t) (void)block_free(ctx, w->q_t, w->block_bytes, w->fence);
         delete w;
         return hip_fail(e, "prepare");
     }
@@ -605,7 +610,7 @@ int32_t mnb_weight_destroy(mnb_weight *w) {
     hipError_t first = hipStreamSynchronize(w->ctx->stream);
     hipError_t e;
     if (w->block_bytes) {
-        if ((e = block_free(w->ctx, w->q_t, w->block_bytes)) != hipSuccess && first == hipSuccess) first = e;
+        if ((e = block_free(w->ctx, w->q_t, w->block_bytes, w->fence)) != hipSuccess && first == hipSuccess) first = e;
     } else {
         if (w->q_t && (e = hipFree(w->q_t)) != hipSuccess && first == hipSuccess) first = e;
         if (w->s_t && (e = hipFree(w->s_t)) != hipSuccess && first == hipSuccess) first = e;

@@ -135,6 +135,7 @@ struct mnb_weight {
     void *zp_t = nullptr;   // tiled zero points (nullptr when implicit 8)
     int64_t bytes = 0;
     size_t block_bytes = 0; // not 0: s_t and zp_t lie in q_t's allocation of this size
+    void *fence = nullptr;  // with block_bytes: a small allocation whose release waits for the device (block_free)
 };
 
 namespace mnb {
