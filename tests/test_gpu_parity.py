@@ -319,6 +319,7 @@ def test_gemm_split_tiles_tails_and_outputs(ctx, M, K, N):
     xd = torch.from_numpy(x16).cuda()
     buf = torch.zeros(M * N + 1, dtype=torch.float32, device="cuda")
     yd = buf[1:]
+    torch.cuda.synchronize()     # the product runs on the context's stream
     w.matmul(xd, yd)
     torch.cuda.synchronize()
     assert np.array_equal(yd.cpu().numpy().reshape(M, N).view(np.uint32), y32.view(np.uint32))
@@ -392,6 +393,7 @@ def test_single_products_k_sliced(ctx, case):
         xd = torch.from_numpy(x16).cuda()
         buf = torch.zeros(M * N + 1, dtype=torch.float32, device="cuda")
         yd = buf[1:]
+        torch.cuda.synchronize()     # the product runs on the context's stream
         w.matmul(xd, yd)
         torch.cuda.synchronize()
         assert np.array_equal(yd.cpu().numpy().reshape(M, N).view(np.uint32), y32.view(np.uint32))
@@ -785,6 +787,7 @@ def test_small_batch_group_with_fp32_scales(ctx):
     g = mnb_hip.Group(ctx, items)
     try:
         assert g.plan().as_tuple() == (STREAM, NO_ORDER, 4, 16), g.plan().as_tuple()
+        torch.cuda.synchronize()     # the group runs on the context's stream
         g.run()
         torch.cuda.synchronize()
         for (w, xd, y), (t, s32, x16) in zip(items, checks):
@@ -988,6 +991,7 @@ def test_single_product_with_x_beyond_2_gib(ctx):
         xd = torch.randn(M, K, device="cuda", generator=gen, dtype=torch.float16)
         assert xd.numel() * 2 > (1 << 31)
         yd = torch.empty(M, N, device="cuda", dtype=torch.float32)
+        torch.cuda.synchronize()     # the products run on the context's stream
         w.matmul(xd, yd)
         yh = torch.empty(M, N, device="cuda", dtype=torch.float16)
         w.matmul(xd, yh)
