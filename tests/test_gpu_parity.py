@@ -1294,6 +1294,35 @@ def test_staged_x_equals_rounded_x(ctx, M, K, offset):
         w.close()
 
 
+@pytest.mark.parametrize("K", [3, 7, 9, 15, 30, 90, 1001, 4099])
+@pytest.mark.parametrize("xt,offset", [("f32", 0), ("f32", 1), ("f16", 0), ("f16", 1), ("f16", 3)])
+def test_staged_rows_of_any_length_and_alignment(ctx, K, xt, offset):
+    """Rows whose ends lie inside a 16-byte piece, at every alignment: the
+    product's bits are those of the weight taken as one of the padded K, on x
+    padded with zeros, which needs no staging."""
+    import torch
+    N, bs = 100, 16
+    Kp = -(-K // bs) * bs
+    t = synth.make_weight(K, N, Kp, bs, with_zp=True)
+    w, wp = (mnb_hip.Weight(ctx, N, k, bs, t.q, t.scales_f16, t.zp_row_padded, mnb_hip.MNB_ZP_ROW_PADDED) for k in (K, Kp))
+    try:
+        for M in (1, 4, 16, 17, 200):
+            g = torch.Generator(device="cuda").manual_seed(K * M)
+            buf = torch.randn((M * K + offset + 8,), generator=g, device="cuda").to(torch.float32 if xt == "f32" else torch.float16)
+            x = buf[offset:offset + M * K].view(M, K)
+            xp = torch.zeros((M, Kp), dtype=torch.float16, device="cuda")
+            xp[:, :K] = x.half()
+            y, ref = torch.empty((M, N), device="cuda"), torch.empty((M, N), device="cuda")
+            torch.cuda.synchronize()
+            w.matmul(x, y)
+            wp.matmul(xp, ref)
+            torch.cuda.synchronize()
+            assert torch.equal(y.view(torch.int32), ref.view(torch.int32)), M
+    finally:
+        w.close()
+        wp.close()
+
+
 @pytest.mark.parametrize("M,K,N,bs,zp,f32s,yt,acc", [
     (193, 896, 9728, 32, False, False, "f16", False),    # one row past three m-tiles
     (200, 896, 9728, 32, True, False, "f32", False),

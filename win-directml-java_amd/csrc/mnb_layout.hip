@@ -10,6 +10,7 @@
 namespace mnb {
 
 typedef u32x4_t u32x4_dq_alias_t __attribute__((may_alias));
+typedef u32x4_t u32x4_row_t __attribute__((may_alias, aligned(2)));   // 16 bytes of a row of fp16 or fp32
 constexpr int kDequantThreads = 256;
 
 WeightGeom make_geom(int32_t N, int32_t K, int32_t bs) {
@@ -206,11 +207,16 @@ hipError_t launch_copy_rows(const WeightGeom &sg, const void *sq, const void *ss
 }
 
 // fp16 copy of x with rows padded to ldx (a multiple of 8).  A launch-bound
-// copy: one thread per 8 values of a row with 16-byte accesses where x's rows
-// are aligned (VEC), and 32-bit index arithmetic unless x has 2^32 pieces or
-// more.  Eight Phi-3 products of 200 fp32 rows in a graph: 295.8 -> 288.7 us
-// against one value per thread with 64-bit divisions.
-template <typename XT, bool VEC, typename IdxT>
+// copy: one thread per 8 values of a row, read in 16-byte pieces at whatever
+// alignment x's rows have, and 32-bit index arithmetic unless x has 2^32
+// pieces or more.  A row's last piece is read so that it ends at the row's
+// end and shifted into place.  Whole products with their staging, same box,
+// one value per thread -> this: 3072 -> 3072 at M = 200 from aligned fp32
+// 17.0 -> 15.4 us, from fp32 off by one 17.0 -> 15.5; 8190 -> 512 at M = 512
+// from fp32 22.0 -> 19.5; 3076 -> 1024 at M = 2048 from fp16 44.7 -> 36.4;
+// 1001 -> 1024 at M = 4 4.7 -> 4.7.  (Eight element loads per thread where a
+// row is unaligned took 24.9 us of the third and 5.2 of the last.)
+template <typename XT, typename IdxT>
 __global__ __launch_bounds__(256) void stage_x_kernel(const XT *__restrict__ x, IdxT pieces, int32_t K, int32_t ldx,
                                                       _Float16 *__restrict__ out) {
     const IdxT e = (IdxT)blockIdx.x * 256 + threadIdx.x;
@@ -218,42 +224,41 @@ __global__ __launch_bounds__(256) void stage_x_kernel(const XT *__restrict__ x, 
     const IdxT per_row = (IdxT)(ldx / 8);
     const IdxT m = e / per_row;
     const int k = (int)(e - m * per_row) * 8;
-    const XT *xp = x + (size_t)m * K + k;
+    const XT *row = x + (size_t)m * K;
     half8_t h;
-    if constexpr (VEC) {   // K == ldx
+    if (K >= 8) {
+        const int kc = min(k, K - 8);
         XT v[8];
-        u32x4_t raw[sizeof(XT) / 2];
+        u32x4_row_t raw[sizeof(XT) / 2];
 #pragma unroll
-        for (int i = 0; i < (int)sizeof(XT) / 2; ++i) raw[i] = gld((const u32x4_t *)xp + i);
+        for (int i = 0; i < (int)sizeof(XT) / 2; ++i)
+            raw[i] = ((const __attribute__((address_space(1))) u32x4_row_t *)(row + kc))[i];
         __builtin_memcpy(v, raw, sizeof v);
 #pragma unroll
         for (int i = 0; i < 8; ++i) h[i] = (_Float16)v[i];
+        if (kc != k) h = __builtin_bit_cast(half8_t, __builtin_bit_cast(unsigned __int128, h) >> (16 * (k - kc)));
     } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) h[i] = k + i < K ? (_Float16)xp[i] : (_Float16)0.0f;
+        for (int i = 0; i < 8; ++i) h[i] = i < K ? (_Float16)row[i] : (_Float16)0.0f;
     }
     *(half8_t *)(out + (size_t)m * ldx + k) = h;
 }
 
-template <typename XT, bool VEC>
+template <typename XT>
 static hipError_t stage_x_typed(const XT *x, int32_t M, int32_t K, int32_t ldx, _Float16 *out, hipStream_t stream) {
     const uint64_t pieces = (uint64_t)M * (uint64_t)(ldx / 8);
     const dim3 grid(blocks_for(pieces, 256)), block(256);
     if (pieces <= 0xFFFFFF00u)
-        hipLaunchKernelGGL((stage_x_kernel<XT, VEC, uint32_t>), grid, block, 0, stream, x, (uint32_t)pieces, K, ldx, out);
+        hipLaunchKernelGGL((stage_x_kernel<XT, uint32_t>), grid, block, 0, stream, x, (uint32_t)pieces, K, ldx, out);
     else
-        hipLaunchKernelGGL((stage_x_kernel<XT, VEC, uint64_t>), grid, block, 0, stream, x, pieces, K, ldx, out);
+        hipLaunchKernelGGL((stage_x_kernel<XT, uint64_t>), grid, block, 0, stream, x, pieces, K, ldx, out);
     return hipGetLastError();
 }
 
 hipError_t launch_stage_x(const void *x, int32_t x_type, int32_t M, int32_t K, int32_t ldx, _Float16 *out,
                           hipStream_t stream) {
-    const bool vec = K == ldx && (uintptr_t)x % 16 == 0;
-    if (x_type == MNB_F32)
-        return vec ? stage_x_typed<float, true>((const float *)x, M, K, ldx, out, stream)
-                   : stage_x_typed<float, false>((const float *)x, M, K, ldx, out, stream);
-    return vec ? stage_x_typed<_Float16, true>((const _Float16 *)x, M, K, ldx, out, stream)
-               : stage_x_typed<_Float16, false>((const _Float16 *)x, M, K, ldx, out, stream);
+    return x_type == MNB_F32 ? stage_x_typed((const float *)x, M, K, ldx, out, stream)
+                             : stage_x_typed((const _Float16 *)x, M, K, ldx, out, stream);
 }
 
 // w = float(q - zp) * scale, formed as (float(q - zp) * stored scale) *
