@@ -241,3 +241,42 @@ def test_quantized_weight_destroyed_during_a_capture(mode, other_thread):
     w.close()
     del graph
     ctx.close()
+
+
+def test_capture_of_fp32_x_before_any_staging():
+    """fp32 x of 16 rows at K = 8320, whose fp16 copy the context has no room
+    for yet: the product is captured all the same (x read in place), and the
+    replays equal the eager products, which stage x, bit for bit; so does a
+    capture made after them."""
+    import torch
+    ctx = mnb_hip.Context(0)
+    M, K, N = 16, 8320, 200
+    w = _weight(ctx, 21, N, K, zp=True)
+    x = torch.empty((M, K), device="cuda")
+    ys = [torch.empty((M, N), device="cuda") for _ in range(3)]
+    st = torch.cuda.Stream()
+    graphs = [torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()]
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graphs[0], stream=st):
+        w.matmul(x, ys[0], stream=st.cuda_stream)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        with torch.cuda.stream(st):
+            x.copy_(torch.randn((M, K), generator=torch.Generator("cuda").manual_seed(rep), device="cuda"))
+            w.matmul(x, ys[2], stream=st.cuda_stream)
+        if rep == 0:
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graphs[1], stream=st):
+                w.matmul(x, ys[1], stream=st.cuda_stream)
+            torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            ys[0].fill_(float("nan"))
+            ys[1].fill_(float("nan"))
+            graphs[0].replay()
+            graphs[1].replay()
+        torch.cuda.synchronize()
+        assert torch.isfinite(ys[2]).all()
+        assert torch.equal(ys[0], ys[2]) and torch.equal(ys[1], ys[2])
+    del graphs
+    w.close()
+    ctx.close()

@@ -779,18 +779,35 @@ size_t mnb::stage_x_limit(const mnb_weight *w, int32_t M, const void *x, int32_t
     return (size_t)M * (size_t)((g.K + 7) & ~7) * 2;
 }
 
-// fp32 x is read in place by the GEMV: a staging launch before it costs 2-4 us,
-// as much as a small product itself (figures at gemv_tile).  The other kernels
-// read x many times and take it from a staged fp16 copy.
-size_t mnb::stage_x_bytes(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, const void *y,
-                          int32_t y_type) {
+bool mnb::can_read_f32_x(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, const void *y,
+                         int32_t y_type) {
     const WeightGeom &g = w->g;
     const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)M * g.K * 4;
     const uintptr_t y0 = (uintptr_t)y, y1 = y0 + (size_t)M * g.N * dtype_size(y_type);
     const bool overlap = y && x0 < y1 && y0 < x1;
-    if (x_type == MNB_F32 && !overlap && (g.K % 8) == 0 && ((uintptr_t)x & 15u) == 0 && M <= mnb::kSkinnyMaxM &&
-        mnb::ks_skinny_plan(g, M, cu_count).wgs == 0)
-        return 0;
+    return x_type == MNB_F32 && !overlap && (g.K % 8) == 0 && ((uintptr_t)x & 15u) == 0 && M <= mnb::kSkinnyMaxM &&
+           mnb::ks_skinny_plan(g, M, cu_count).wgs == 0;
+}
+
+// fp32 x is read in place by the GEMV where that costs less than the staging
+// launch it saves (1.8-2 us).  Every workgroup (n-tile) reads all of x, at
+// twice the bytes of staged x, and a CU gets those at about 90 KB/us from L2:
+// the extra 2 M K bytes of each of its rounds of workgroups pay up to about
+// 96 Ki values of x per CU (staged / in place, us, fp32 y, bs 32: 3072 -> 16384
+// at M = 5 10.4 / 9.9; 3072 -> 32064 at M = 3 15.1 / 14.3, 5 16.3 / 17.4, 8 18.0 /
+// 19.6; 8192 -> 3072 at M = 8 8.5 / 8.1, 12 9.9 / 10.2; 8192 -> 28672 at M = 4
+// 28.4 / 30.9, 8 33.6 / 40.3; 896 -> 151936 at M = 8 20.7 / 25.9, 16 30.1 /
+// 42.7).  At M <= 2 the weight stream hides them on every shape timed (896 ->
+// 151936 at M = 2 17.0 / 16.7, 8192 -> 28672 27.2 / 26.5).
+constexpr int64_t kF32XRowElems = 96 * 1024;
+
+size_t mnb::stage_x_bytes(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, const void *y,
+                          int32_t y_type) {
+    if (can_read_f32_x(w, cu_count, M, x, x_type, y, y_type)) {
+        const int64_t cu = cu_count > 0 ? cu_count : 256;
+        const int64_t rounds = (w->g.NT + cu - 1) / cu;
+        if (M <= 2 || rounds * M * w->g.K < kF32XRowElems) return 0;
+    }
     return stage_x_limit(w, M, x, x_type);
 }
 
@@ -813,7 +830,7 @@ hipError_t mnb::launch_product(const mnb_weight *w, int cu_count, int32_t M, con
                                hipStream_t s) {
     const WeightGeom &g = w->g;
     const int32_t ldx_pad = (g.K + 7) & ~7;
-    if (stage_x_bytes(w, cu_count, M, x, x_type, y, y_type) != 0) {
+    if (stage_x) {
         const hipError_t e = mnb::launch_stage_x(x, x_type, M, g.K, ldx_pad, (_Float16 *)stage_x, s);
         if (e != hipSuccess) return e;
         return launch_staged(w, cu_count, M, (const _Float16 *)stage_x, ldx_pad, y, y_type, accumulate, sk_ws, ws_bytes, s);
@@ -890,7 +907,15 @@ int32_t mnb_matmul(mnb_context *ctx, const mnb_weight *w, int32_t M, const void 
             return hip_fail(e, op);
         xd = *buf;
     }
-    const size_t stage = mnb::stage_x_bytes(w, ctx->cu_count, M, xd, x_type, host ? nullptr : y, y_type);
+    size_t stage = mnb::stage_x_bytes(w, ctx->cu_count, M, xd, x_type, host ? nullptr : y, y_type);
+    if (stage > ctx->stage_x_cap && !host &&
+        mnb::can_read_f32_x(w, ctx->cu_count, M, xd, x_type, y, y_type)) {
+        // nothing may be allocated in a stream capture: x is read in place
+        // there (the same bits) when no earlier call has left room for it
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(s, &cs) != hipSuccess) (void)hipGetLastError();
+        if (cs != hipStreamCaptureStatusNone) stage = 0;
+    }
     if (stage && (e = ensure(ctx, &ctx->stage_x, &ctx->stage_x_cap, stage)) != hipSuccess) return hip_fail(e, op);
 
     void *yd = y;
@@ -903,8 +928,8 @@ int32_t mnb_matmul(mnb_context *ctx, const mnb_weight *w, int32_t M, const void 
             return hip_fail(e, op);
     }
 
-    e = mnb::launch_product(w, ctx->cu_count, M, xd, x_type, yd, y_type, (flags & MNB_ACCUMULATE) != 0, ctx->stage_x,
-                            ctx->sk_ws, ctx->sk_ws_cap, s);
+    e = mnb::launch_product(w, ctx->cu_count, M, xd, x_type, yd, y_type, (flags & MNB_ACCUMULATE) != 0,
+                            stage ? ctx->stage_x : nullptr, ctx->sk_ws, ctx->sk_ws_cap, s);
     if (e != hipSuccess) return hip_fail(e, op);
 
     if (host) {

@@ -318,10 +318,14 @@ ProductPlan product_plan(const WeightGeom &g, int32_t M, int32_t cu_count);
 // status, with the message recorded.
 int32_t check_matmul(const mnb_context *ctx, const mnb_weight *w, int32_t M, const void *x, int32_t x_type,
                      int64_t x_elems, const void *y, int32_t y_type, int64_t y_elems, uint32_t flags);
-// Bytes of staged fp16 x a product needs: 0 when the kernels read x in place,
-// i.e. x is 16-byte aligned, K is a multiple of 8, and x is fp16 or the
-// product runs on the GEMV, which rounds fp32 x itself (unless y overlaps x:
-// a staged fp32 x may be overwritten by its product); else M rows of K rounded
+// Whether the GEMV can read this x in place and round it itself: 16-byte
+// aligned fp32, K a multiple of 8, a product that runs on the GEMV, and no y
+// that overlaps x (a staged fp32 x may be overwritten by its product).
+bool can_read_f32_x(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, const void *y,
+                    int32_t y_type);
+// Bytes of staged fp16 x a product is given: 0 when x is read in place, i.e.
+// 16-byte aligned fp16 with K a multiple of 8, or fp32 that can_read_f32_x
+// allows and that is cheaper to read than to stage; else M rows of K rounded
 // up to 8.
 size_t stage_x_bytes(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, const void *y,
                      int32_t y_type);
@@ -331,8 +335,8 @@ size_t stage_x_limit(const mnb_weight *w, int32_t M, const void *x, int32_t x_ty
 // sk_workspace_bytes(G) over the stream-K grids of its row chunks (0 when no
 // chunk runs stream-K).
 size_t prefill_workspace_bytes(const WeightGeom &g, int32_t M, int32_t cu_count);
-// One product on device pointers: x staged into stage_x when stage_x_bytes
-// says so, then the GEMV (M <= 16) or the GEMM, whose split tiles use
+// One product on device pointers: x staged into stage_x unless that is null
+// (which stage_x_bytes == 0 or can_read_f32_x allows), then the GEMV (M <= 16) or the GEMM, whose split tiles use
 // sk_ws (ws_bytes bytes, at least sk_workspace_bytes(sk_max_grid(cu_count))).
 // Allocates nothing.
 hipError_t launch_product(const mnb_weight *w, int cu_count, int32_t M, const void *x, int32_t x_type, void *y,

@@ -79,8 +79,9 @@ extern "C" int32_t mnb_matmul_noalloc(mnb_context *ctx, const mnb_weight *w, int
     mnb::DeviceGuard guard(ctx->device);
     hipStream_t s = stream ? (hipStream_t)stream : ctx->stream;
     unsigned char *base = (unsigned char *)ctx->scratch;
+    const bool staged = mnb::stage_x_bytes(w, ctx->cu_count, M, x, x_type, y, y_type) != 0;
     const hipError_t e = mnb::launch_product(w, ctx->cu_count, M, x, x_type, y, y_type, (flags & MNB_ACCUMULATE) != 0,
-                                             base + kWorkspaceBytes, base, kWorkspaceBytes, s);
+                                             staged ? base + kWorkspaceBytes : nullptr, base, kWorkspaceBytes, s);
     if (e != hipSuccess) {
         snprintf(msg, sizeof msg, "MatMulNBitsKernel.%s failed: %s (%s)", M == 1 ? "matvec" : "matmulBatch",
                  hipGetErrorString(e), hipGetErrorName(e));
