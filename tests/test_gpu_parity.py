@@ -1369,6 +1369,47 @@ def test_single_products_on_64_row_tiles(ctx, M, K, N, bs, zp, f32s, yt, acc):
         w.close()
 
 
+@pytest.mark.parametrize("K", [100, 256, 384, 500, 640, 768, 896, 1024])   # one to eight waves
+@pytest.mark.parametrize("M,N,zp,yt,acc", [(17, 200, True, "f16", False), (100, 1500, False, "f32", True),
+                                           (200, 2050, True, "f32", False), (33, 9728, False, "f16", True),
+                                           (40, 16001, True, "f32", False)])
+def test_k_sliced_workgroups_of_one_to_eight_waves(ctx, M, K, N, zp, yt, acc):
+    """K-sliced products at every number of waves a workgroup can have, whose
+    LDS and sum depend on it (several workgroups share a CU with the fewest),
+    with 32 x 16 to 48 x 64 blocks, against a float32 product of the
+    dequantized weight, and the same bits again."""
+    import torch
+    t = synth.make_weight(M + K, N, K, 32, with_zp=zp)
+    w = mnb_hip.Weight(ctx, N, K, 32, t.q, t.scales_f16, t.zp_row_padded if zp else None,
+                       mnb_hip.MNB_ZP_ROW_PADDED if zp else None)
+    try:
+        assert w.plan(M).kernel == KSLICE, w.plan(M).as_tuple()
+        td = torch.float32 if yt == "f32" else torch.float16
+        g = torch.Generator(device="cuda").manual_seed(M + K)
+        x = torch.randn((M, K), generator=g, device="cuda").half()
+        y0 = torch.randn((M, N), generator=g, device="cuda").to(td)
+        wd = torch.empty((N, K), dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        w.dequantize(out=wd)
+        torch.cuda.synchronize()
+        ref = x.float() @ wd.t().contiguous()
+        if acc:
+            ref += y0.float()
+        bound = 1e-3 * K ** 0.5 * float(x.abs().max()) * float(wd.abs().max())
+        bound = bound + (ref.abs() * 2.0 ** -10 if yt == "f16" else 0.0)   # one fp16 ulp
+        runs = []
+        for _ in range(2):
+            y = y0.clone()
+            torch.cuda.synchronize()
+            w.matmul(x, y, accumulate=acc)
+            torch.cuda.synchronize()
+            runs.append(y)
+        assert torch.equal(runs[0], runs[1])
+        assert bool(((runs[0].float() - ref).abs() <= bound).all())
+    finally:
+        w.close()
+
+
 @pytest.mark.parametrize("M,K,N,bs,zp,yt,acc", [
     (33, 3072, 9216, 32, False, "f16", False),   # the fewest rows of one block
     (48, 3000, 9215, 128, True, "f32", True),    # a whole block; N and K end inside a tile

@@ -31,6 +31,7 @@
 // super-tiles loaded at once into LDS slower: at these sizes a workgroup is
 // bound by its CU's issue of dequantization, LDS passes and MFMAs.)
 #include <algorithm>
+#include <type_traits>
 
 #include "mnb_device.h"
 
@@ -45,8 +46,8 @@ __global__ __launch_bounds__(64 * kKsMaxWaves) void gemm_ks_kernel(KsParams p) {
     constexpr int ZB = SPS <= 2 ? 1 : SPS / 2;
     constexpr int U = MB * NTW;
     // wave-private x blocks in the main loop; the reduction reuses the space
-    // for the waves' partial blocks (U 16x16 units of 1 KiB each)
-    __shared__ __align__(16) unsigned char smem[kKsMaxWaves * (U > 4 ? U : 4) * 1024];
+    // for the waves' partial blocks (ks_lds_bytes)
+    extern __shared__ __align__(16) unsigned char smem[];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -178,37 +179,15 @@ __global__ __launch_bounds__(64 * kKsMaxWaves) void gemm_ks_kernel(KsParams p) {
         }
     }
 
-    // Sum the waves' partial blocks: every wave writes its U units to LDS,
-    // then unit q is summed over waves 0..W-1 (in that order) and stored by
-    // wave q mod W.  One round, with a unit's W loads in flight together: in
-    // rounds of four units on four of the eight waves, one load after
-    // another, this cost a 64 x 64 block 1 us more (same box: 896 -> 9728 at
-    // M = 37 8.2 -> 7.1 us, 3072 -> 16384 at M = 37 14.1 -> 12.9, 3072 -> 9216
-    // at M = 128 24.9 -> 23.1, 3072 -> 3072 at M = 200 13.7 -> 12.5; the
-    // smaller blocks 0-2%).
-    __syncthreads();   // every wave is done with its x block
-    float4_ks_alias_t *red = (float4_ks_alias_t *)smem;
+    // y's rows and columns of this lane.  The lane is counted anew here, so
+    // that its parts hold no registers through the main loop.
+    const int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u)), er = el & 15, eg = el >> 4;
     const int n_grp = ng * NTW * kTileRows;
-#pragma unroll
-    for (int q = 0; q < U; ++q) red[(wave * U + q) * 64 + lane] = acc[q / NTW][q % NTW];
-    __syncthreads();
-    for (int q = wave; q < U; q += W) {
-        float4_t o[kKsMaxWaves];
-#pragma unroll
-        for (int w2 = 0; w2 < kKsMaxWaves; ++w2) o[w2] = red[(min(w2, W - 1) * U + q) * 64 + lane];
-        float4_t v = o[0];
-#pragma unroll
-        for (int w2 = 1; w2 < kKsMaxWaves; ++w2)
-            if (w2 < W) {
-                v[0] += o[w2][0];
-                v[1] += o[w2][1];
-                v[2] += o[w2][2];
-                v[3] += o[w2][3];
-            }
-        // unit (b, t): lane (gg, r) holds row m0 + 16 b + r, columns n .. n + 3
+    auto store_unit = [&](int q, float4_t v) __attribute__((always_inline)) {
+        // unit (b, t): lane (eg, er) holds row m0 + 16 b + er, columns n .. n + 3
         const int b = q / NTW, t = q % NTW;
-        const int m = m0 + 16 * b + r;
-        const int n = n_grp + t * kTileRows + 4 * gg;
+        const int m = m0 + 16 * b + er;
+        const int n = n_grp + t * kTileRows + 4 * eg;
         if (m < p.M && n < p.N) {
             // undo the stored scales' factor 2^fold_exp (exact)
             v[0] *= p.unfold;
@@ -249,14 +228,75 @@ __global__ __launch_bounds__(64 * kKsMaxWaves) void gemm_ks_kernel(KsParams p) {
                     }
             }
         }
+    };
+
+    // Sum the waves' partial blocks: every wave writes its U units to LDS,
+    // then unit q is summed over waves 0..W-1 (in that order) and stored by
+    // wave q mod W.  One round, with exactly the unit's W loads in flight
+    // together.  Against rounds of four units on four waves, one load after
+    // another (same box, block forced, us): 64 x 64 3072 -> 3072 at M = 64 13.2
+    // -> 11.6, 896 -> 9728 8.3 -> 7.2, 3072 -> 9216 at M = 200 40.4 -> 35.0;
+    // 32 x 64 3072 -> 3072 at M = 64 9.2 -> 8.6; 32 x 32 7.2 -> 7.0, 3072 -> 9216
+    // at M = 200 45.2 -> 41.2; 32 x 16 8.8 -> 8.7 (3% slower where it runs
+    // many rounds, which it is not chosen for).  Loading as many units as the
+    // largest workgroup has waves, whatever W is, cost short K up to a
+    // quarter (32 x 64, 128 -> 4096 4.6 -> 5.8, 256 -> 4096 4.4 -> 5.0); one wave
+    // alone stores its block as it is (4.1).
+    if (W == 1) {
+#pragma unroll
+        for (int q = 0; q < U; ++q) store_unit(q, acc[q / NTW][q % NTW]);
+        return;
     }
+    __syncthreads();   // every wave is done with its x block
+    float4_ks_alias_t *red = (float4_ks_alias_t *)smem;
+#pragma unroll
+    for (int q = 0; q < U; ++q) red[(wave * U + q) * 64 + el] = acc[q / NTW][q % NTW];
+    __syncthreads();
+    for (int q = wave; q < U; q += W) {
+        float4_t v = {0.f, 0.f, 0.f, 0.f};
+        auto sum = [&](auto waves) __attribute__((always_inline)) {
+            constexpr int NW = decltype(waves)::value;
+            float4_t o[NW];
+#pragma unroll
+            for (int w2 = 0; w2 < NW; ++w2) o[w2] = red[(w2 * U + q) * 64 + el];
+            v = o[0];
+#pragma unroll
+            for (int w2 = 1; w2 < NW; ++w2) {
+                v[0] += o[w2][0];
+                v[1] += o[w2][1];
+                v[2] += o[w2][2];
+                v[3] += o[w2][3];
+            }
+        };
+        switch (W) {
+            case 2: sum(std::integral_constant<int, 2>{}); break;
+            case 3: sum(std::integral_constant<int, 3>{}); break;
+            case 4: sum(std::integral_constant<int, 4>{}); break;
+            case 5: sum(std::integral_constant<int, 5>{}); break;
+            case 6: sum(std::integral_constant<int, 6>{}); break;
+            case 7: sum(std::integral_constant<int, 7>{}); break;
+            default: sum(std::integral_constant<int, kKsMaxWaves>{}); break;
+        }
+        store_unit(q, v);
+    }
+}
+
+// LDS of a workgroup of `waves` waves: a 4 KiB x block or the U 16x16 units
+// of 1 KiB of its output block per wave, whichever is larger.  By the waves
+// there are, not by kKsMaxWaves: with four or fewer (K <= 512) the registers let
+// two to eight workgroups share a CU, and so must the LDS (room for eight
+// waves / for those there are, us: 48 x 64, 128 -> 4096 at M = 200 13.0 / 7.9;
+// 64 x 64, 384 -> 9728 at M = 128 12.2 / 8.3).
+static unsigned ks_lds_bytes(int mb, int ntw, unsigned waves) {
+    return waves * 1024u * (unsigned)std::max(mb * ntw, 4);
 }
 
 template <typename ScaleT, bool HAS_ZP, int SPS>
 static hipError_t ks_shape(const KsConfig &c, dim3 grid, dim3 block, hipStream_t s, const KsParams &p) {
 #define MNB_KS(MB_, NTW_)                                                                               \
     if (c.mb == MB_ && c.ntw == NTW_) {                                                                 \
-        hipLaunchKernelGGL((gemm_ks_kernel<ScaleT, HAS_ZP, SPS, MB_, NTW_>), grid, block, 0, s, p);     \
+        hipLaunchKernelGGL((gemm_ks_kernel<ScaleT, HAS_ZP, SPS, MB_, NTW_>), grid, block,               \
+                           ks_lds_bytes(MB_, NTW_, block.x / 64), s, p);                                \
         return hipGetLastError();                                                                       \
     }
     MNB_KS(1, 4)
