@@ -8,7 +8,10 @@
 //   "grid", "split" and "parts": see check_grid, check_split, check_parts;
 //   K-sliced plan of single products (mnb::ks_single_plan): the word
 //   "ksplan", then lines "M NT ST scale_f32 has_zp sps", each answered with
-//   "mb ntw est wgs" (mb 0: no supported block).
+//   "mb ntw est wgs" (mb 0: no supported block);
+//   whole plan of single products (mnb::single_product_plan): the word "plan",
+//   then the same lines, each answered with "ks rows cols G" (ks 1: K-sliced;
+//   the output tile's rows and columns; the workgroups).
 // Exits 1 on the first broken invariant; prints balance (and, for the tile
 // list, locality) figures.
 #include <stdio.h>
@@ -328,6 +331,18 @@ static int print_ksplan() {
     return 0;
 }
 
+static int print_plan() {
+    int M, NT, ST, f32, zp, sps;
+    while (scanf("%d %d %d %d %d %d", &M, &NT, &ST, &f32, &zp, &sps) == 6) {
+        const ProductPlan p = single_product_plan(M, NT, ST, f32, zp, sps, 256);
+        if (p.ks && !ks_config_supported(p.kc.mb, p.kc.ntw, f32, zp, sps)) return fail("plan block", p.kc.mb, p.kc.ntw);
+        if (!p.ks && (p.sp.G < 1 || p.sp.G > kSkMaxGrid)) return fail("plan grid", M, p.sp.G);
+        if (p.ks) printf("1 %d %d %lld\n", 16 * p.kc.mb, 16 * p.kc.ntw, (long long)ks_workgroups(M, NT, p.kc));
+        else printf("0 %d %d %d\n", 32 * p.sp.fm, 128 * p.sp.ntw, p.sp.G);
+    }
+    return 0;
+}
+
 int main() {
     char first[32] = {0};
     if (scanf("%31s", first) != 1) return fail("input", 0, 0);
@@ -337,6 +352,7 @@ int main() {
     if (strcmp(first, "split") == 0) return check_split();
     if (strcmp(first, "parts") == 0) return check_parts();
     if (strcmp(first, "ksplan") == 0) return print_ksplan();
+    if (strcmp(first, "plan") == 0) return print_plan();
     const int G = atoi(first);
     if (G < 1) return fail("input", G, 0);
     std::vector<SkItem> items;

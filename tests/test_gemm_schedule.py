@@ -315,3 +315,65 @@ def test_k_sliced_plan_respects_supported_blocks(checker):
         assert mb in (2, 4) and est > 0
         if mb == 4:
             assert bs != 16 and not (f32 and zp), (M, K, N, f32, zp, bs)
+
+
+def single_plan(checker, queries):
+    """mnb::single_product_plan for (M, K, N, scale_f32, has_zp, bs) queries:
+    [(K-sliced, tile rows, tile columns, workgroups)]."""
+    lines = []
+    for M, K, N, f32, zp, bs in queries:
+        kpad = -(-K // bs) * bs
+        lines.append("%d %d %d %d %d %d" % (M, -(-N // 16), -(-kpad // 128), f32, zp, 128 // bs))
+    r = subprocess.run([checker], input="plan\n" + "\n".join(lines) + "\n", capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
+    out = [tuple(int(v) for v in line.split()) for line in r.stdout.strip().splitlines()]
+    assert len(out) == len(queries)
+    return out
+
+
+def test_64_row_tiles_by_variant_and_length(checker):
+    """Where single products run on 64 x 256 tiles: the form of each product is
+    the faster of those timed on MI355X (us, same box: 64 x 256 tiles, then
+    split (G over the 128-row tiles) or whole 128 x 256 tiles, or the K-sliced
+    kernel's best block)."""
+    half, gemm, ks = (0, 64, 256), (0, 128, 256), 1
+    cases = [  # (M, K, N, fp32 scales, zero points, bs) -> form
+        ((256, 3072, 9216, 0, 0, 32), half),      # 30.4; split 31.8
+        ((256, 3072, 9216, 0, 1, 64), gemm),      # 34.2; split 33.1
+        ((256, 3072, 9216, 0, 1, 128), gemm),     # 34.4; split 33.3
+        ((256, 3072, 9216, 1, 0, 32), gemm),      # 39.1; split 33.1
+        ((256, 3072, 9216, 1, 1, 128), gemm),     # 41.2; split 34.7
+        ((700, 3072, 3072, 0, 0, 32), half),      # 30.1; split 31.5
+        ((700, 3072, 3072, 1, 1, 32), gemm),      # 41.6; split 33.7
+        ((100, 3072, 16384, 0, 1, 16), gemm),     # 35.0; split 29.5
+        ((384, 3072, 9216, 0, 0, 32), half),      # 34.1; whole 40.6
+        ((384, 3072, 9216, 1, 1, 16), half),      # 44.0; whole 52.7
+        ((1024, 3072, 3072, 0, 1, 128), half),    # 34.7; whole 45.3
+        ((200, 896, 9728, 1, 1, 32), half),       # 18.0; whole 21.4
+        ((200, 3072, 9216, 0, 0, 32), half),      # 30.2; K-sliced 37.6
+        ((632, 256, 2960, 0, 0, 32), ks),         # 8.9; K-sliced 6.5
+        ((33, 256, 27408, 0, 0, 32), ks),         # 8.2; K-sliced 7.0
+        ((52, 192, 24736, 0, 0, 16), ks),         # 8.6; K-sliced 7.0
+        ((336, 288, 9528, 0, 0, 32), half),       # 10.7; K-sliced 14.3
+    ]
+    for (q, want), got in zip(cases, single_plan(checker, [q for q, _ in cases])):
+        assert got[0] == 1 if want == ks else got[:3] == want, (q, got, want)
+
+
+def test_single_product_plan_is_one_of_the_compiled_forms(checker):
+    """Over random shapes and every weight variant: a compiled K-sliced block
+    (no 48- or 64-row one with bs 16 or with fp32 scales and zero points), or
+    128 x 256, 64 x 256 or (where compiled) 128 x 512 GEMM tiles on 1 to 256
+    workgroups."""
+    rng = np.random.default_rng(43)
+    queries = []
+    for _ in range(3000):
+        queries.append((int(rng.integers(17, 2049)), int(rng.integers(8, 20000)), int(rng.integers(1, 200000)),
+                        int(rng.integers(0, 2)), int(rng.integers(0, 2)), int(rng.choice([16, 32, 64, 128]))))
+    for (M, K, N, f32, zp, bs), (ks, rows, cols, wgs) in zip(queries, single_plan(checker, queries)):
+        if ks:
+            assert (rows, cols) in ((32, 16), (32, 32), (32, 64), (48, 64), (64, 64))
+            assert rows == 32 or (bs != 16 and not (f32 and zp)), (M, K, N, f32, zp, bs)
+            assert wgs == -(-N // cols) * -(-M // rows)
+        else:
+            assert (rows, cols) in ((128, 256), (64, 256), (128, 512)) and 1 <= wgs <= 256

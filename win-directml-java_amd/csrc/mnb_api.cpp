@@ -682,33 +682,8 @@ int32_t mnb_max_batch_rows(void) { return std::numeric_limits<int32_t>::max() / 
 
 }  // extern "C"
 
-constexpr double kHalfMargin = 0.95;
-
 mnb::ProductPlan mnb::product_plan(const WeightGeom &g, int32_t M, int32_t cu_count) {
-    ProductPlan p;
-    p.sp = sk_single_plan(M, g.NT, g.ST, g.scale_f32, g.SPS, cu_count);
-    const KsPlan k = ks_single_plan(M, g.NT, g.ST, g.scale_f32, g.has_zp, g.SPS, cu_count);
-    p.ks = k.wgs > 0 && k.est < p.sp.est;
-    p.kc = k.c;
-    // 64 x 256 tiles where they are expected to beat both by more than the
-    // models' error
-    const SinglePlan h = sk_half_plan(M, g.NT, g.ST, cu_count);
-    if (h.est < kHalfMargin * (p.ks ? k.est : p.sp.est)) {
-        p.ks = false;
-        p.sp = h;
-    }
-    // 48-row blocks where they take no more rounds of workgroups than 64-row
-    // ones: a block loads, turns and multiplies a quarter less of x (us, same
-    // box, 64 -> 48 rows.  As many blocks: 3072 -> 9216 at M = 48 12.2 -> 11.0
-    // and 140 25 -> 21.1, 3072 -> 16384 at M = 48 12.9 -> 11.8, 896 -> 9728 at
-    // M = 48 7.1 -> 6.5.  More blocks, as many rounds: 3072 -> 3072 at M = 200
-    // 12.5 -> 11.6 and 400 23.2 -> 21.6, 8192 -> 3072 at M = 200 25.4 -> 23.1).
-    if (p.ks && p.kc.mb == 4 && p.kc.ntw == 4) {
-        const int64_t cu = cu_count > 0 ? cu_count : 256;
-        const KsConfig c48{3, 4};
-        if ((ks_workgroups(M, g.NT, c48) + cu - 1) / cu <= (ks_workgroups(M, g.NT, p.kc) + cu - 1) / cu) p.kc = c48;
-    }
-    return p;
+    return single_product_plan(M, g.NT, g.ST, g.scale_f32, g.has_zp, g.SPS, cu_count);
 }
 
 size_t mnb::prefill_workspace_bytes(const WeightGeom &g, int32_t M, int32_t cu_count) {

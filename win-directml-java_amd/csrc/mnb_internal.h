@@ -300,18 +300,11 @@ struct KsParams {
     float unfold;                      // 2^-fold_exp of the weight
 };
 hipError_t launch_gemm_ks(const mnb_weight *w, const MatmulArgs &a, const KsConfig &c, hipStream_t stream);
-// How one product (one chunk of at most 2 GiB of x rows, M > 16) runs: the
-// K-sliced kernel when its cost model expects it to finish before the GEMM's
-// plan, else that plan.
 // How one product with M <= 16 runs: for 9 <= M <= 16 the K-sliced kernel
 // with 16-row blocks where its cost model expects it to beat the GEMV's by a
 // margin, else the GEMV (wgs == 0).
 KsPlan ks_skinny_plan(const WeightGeom &g, int32_t M, int32_t cu_count);
-struct ProductPlan {
-    bool ks;
-    KsConfig kc;
-    SinglePlan sp;
-};
+// How one product (one chunk of at most 2 GiB of x rows, M > 16) runs.
 ProductPlan product_plan(const WeightGeom &g, int32_t M, int32_t cu_count);
 
 // Argument checks of a product (the reference's messages); MNB_OK or the

@@ -201,7 +201,8 @@ int sk_grid(int T, int ST, int cu_count) {
 
 SinglePlan sk_single_plan(int M, int NT, int ST, int scale_f32, int sps, int cu_count) {
     const int T = sk_tiles(M, NT);
-    SinglePlan plan{false, kGemmNTW, kGemmFM, sk_grid(T, ST, cu_count), 0.0};
+    SinglePlan plan{false, kGemmNTW, kGemmFM, sk_grid(T, ST, cu_count), 0.0, 0};
+    plan.stages = ((int64_t)T * ST + plan.G - 1) / plan.G;
     const double stream_k = sk_cost(T, ST, plan.G, cu_count);
     plan.est = stream_k;
     if (!sk_wide_supported(scale_f32, sps)) return plan;
@@ -211,7 +212,7 @@ SinglePlan sk_single_plan(int M, int NT, int ST, int scale_f32, int sps, int cu_
     for (int g = 0; g < Gw; ++g) busiest = std::max(busiest, sk_cf_first(Tw, Gw, g + 1) - sk_cf_first(Tw, Gw, g));
     const double load = (double)Gw / cu_count;
     const double wide = busiest * (ST * (kStageUs + kStageBusyUs * load) * kGemmWideStageCost + kTileUs);
-    if (wide < stream_k) plan = SinglePlan{true, kGemmWideNTW, kGemmFM, Gw, wide};
+    if (wide < stream_k) plan = SinglePlan{true, kGemmWideNTW, kGemmFM, Gw, wide, (int64_t)2 * busiest * ST};
     return plan;
 }
 
@@ -231,7 +232,8 @@ SinglePlan sk_half_plan(int M, int NT, int ST, int cu_count) {
     int busiest = 0;
     for (int g = 0; g < G; ++g) busiest = std::max(busiest, sk_cf_first(T, G, g + 1) - sk_cf_first(T, G, g));
     const double load = (double)G / cu_count;
-    return SinglePlan{true, kGemmNTW, kGemmHalfFM, G, 2.5 + busiest * (ST * (0.90 + 0.13 * load) + 3.7 + 3.0 * load)};
+    return SinglePlan{true, kGemmNTW, kGemmHalfFM, G, 2.5 + busiest * (ST * (0.90 + 0.13 * load) + 3.7 + 3.0 * load),
+                      (int64_t)busiest * ST};
 }
 
 }  // namespace mnb
@@ -343,6 +345,63 @@ KsPlan ks_single_plan(int M, int NT, int ST, int scale_f32, int has_zp, int sps,
 
 int64_t ks_workgroups(int M, int NT, const KsConfig &c) {
     return (int64_t)((NT + c.ntw - 1) / c.ntw) * ((M + 16 * c.mb - 1) / (16 * c.mb));
+}
+
+// What scales and zero points add to a 256-column stage's dequantization (us).
+// sk_cost and sk_half_plan are fitted to fp16 scales without zero points;
+// 64-row stages took, beside those of bs 32, at bs 16 / 32 / 64 / 128 (24
+// stages, 144 workgroups): fp16 scales with zero points +0.21 / - / 0.16 /
+// 0.16, fp32 scales without +0.36 (bs 32), with +0.52 / 0.48 / - / 0.45; whole
+// 128-row tiles the same to within 0.06.
+static double variant_stage_us(int scale_f32, int has_zp) {
+    return scale_f32 ? (has_zp ? 0.47 : 0.36) : (has_zp ? 0.18 : 0.0);
+}
+
+// 64 x 256 tiles run where they are expected to beat the other forms by more
+// than the models' error, 5%; 16% against tiles split three or more ways,
+// which sk_cost overrates (3072 -> 9216 at M = 256, 72 tiles on 216 workgroups:
+// 37.6 for 31.8 us measured; 3072 -> 16384 at M = 100 with bs 16: 36.2 for
+// 28.5).  The variant's dequantization counts on both sides: a workgroup with
+// split tiles has fewer stages, so with zero points or fp32 scales those win
+// where plain scales lose (us, 128 x 256 split / 64 x 256, 3072 -> 9216 at M =
+// 256: fp16 scales 31.8 / 30.4, with zero points 33.1 / 34.3, fp32 scales 33.1 /
+// 39.1, with both 34.0 / 41.9; against whole 128 x 256 tiles, at M = 384, from
+// 40.6 / 34.1 to 52.7 / 44.0, 64 x 256 ones win with every variant).  Against the
+// K-sliced kernel, which dequantizes as often, it need not count (at M = 200
+// 37.6 / 30.2 to 50.9 / 42.9); but that kernel's model overrates products of one
+// and two super-tiles (of 11 timed, K 128 to 256 and N 2264 to 27408, its best
+// block was 4-27% faster on every one: 256 -> 2960 at M = 632 6.5 / 8.9; of three
+// with three super-tiles 14-25% slower).
+constexpr double kHalfMargin = 0.95, kHalfSplitMargin = 0.84;
+constexpr int kHalfMinST = 3;
+
+ProductPlan single_product_plan(int M, int NT, int ST, int scale_f32, int has_zp, int sps, int cu_count) {
+    ProductPlan p;
+    p.sp = sk_single_plan(M, NT, ST, scale_f32, sps, cu_count);
+    const KsPlan k = ks_single_plan(M, NT, ST, scale_f32, has_zp, sps, cu_count);
+    p.ks = k.wgs > 0 && k.est < p.sp.est;
+    p.kc = k.c;
+    const SinglePlan h = sk_half_plan(M, NT, ST, cu_count);
+    const double v = variant_stage_us(scale_f32, has_zp);
+    const bool split = !p.sp.closed && p.sp.G >= 3 * (int64_t)sk_tiles(M, NT);
+    const bool beats_gemm =
+        h.est + v * h.stages < (split ? kHalfSplitMargin : kHalfMargin) * (p.sp.est + v * p.sp.stages);
+    if (p.ks ? ST >= kHalfMinST && h.est < kHalfMargin * k.est : beats_gemm) {
+        p.ks = false;   // where 64 x 256 tiles beat it but not the GEMM's other form, that one does too
+        if (beats_gemm) p.sp = h;
+    }
+    // 48-row blocks where they take no more rounds of workgroups than 64-row
+    // ones: a block loads, turns and multiplies a quarter less of x (us, same
+    // box, 64 -> 48 rows.  As many blocks: 3072 -> 9216 at M = 48 12.2 -> 11.0
+    // and 140 25 -> 21.1, 3072 -> 16384 at M = 48 12.9 -> 11.8, 896 -> 9728 at
+    // M = 48 7.1 -> 6.5.  More blocks, as many rounds: 3072 -> 3072 at M = 200
+    // 12.5 -> 11.6 and 400 23.2 -> 21.6, 8192 -> 3072 at M = 200 25.4 -> 23.1).
+    if (p.ks && p.kc.mb == 4 && p.kc.ntw == 4) {
+        const int64_t cu = cu_count > 0 ? cu_count : 256;
+        const KsConfig c48{3, 4};
+        if ((ks_workgroups(M, NT, c48) + cu - 1) / cu <= (ks_workgroups(M, NT, p.kc) + cu - 1) / cu) p.kc = c48;
+    }
+    return p;
 }
 
 }  // namespace mnb

@@ -156,7 +156,8 @@ double sk_cost(int64_t T, int64_t ST, int64_t G, int cu_count);
 struct SinglePlan {
     bool closed;
     int ntw, fm, G;
-    double est;   // the cost model's time (us)
+    double est;       // the cost model's time (us)
+    int64_t stages;   // 256-column stages of the busiest workgroup
 };
 SinglePlan sk_single_plan(int M, int NT, int ST, int scale_f32, int sps, int cu_count);
 // Whole 64 x 256 tiles in closed-form order, and their estimate, for the
@@ -182,6 +183,14 @@ struct KsPlan {
     int64_t wgs;
 };
 KsPlan ks_single_plan(int M, int NT, int ST, int scale_f32, int has_zp, int sps, int cu_count);
+// How one product with M > 16 runs: on the K-sliced kernel (ks) with block kc,
+// or on the GEMM as sp says.
+struct ProductPlan {
+    bool ks;
+    KsConfig kc;
+    SinglePlan sp;
+};
+ProductPlan single_product_plan(int M, int NT, int ST, int scale_f32, int has_zp, int sps, int cu_count);
 
 // The split tiles of one launch, passed by value in the reduce kernel's
 // arguments, so nothing is allocated: tile t of item `item` and its
