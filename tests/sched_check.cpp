@@ -103,6 +103,9 @@ static int check_closed() {
         std::vector<SkTile> seq;
         std::vector<SkRange> wg;
         sk_tile_list(items, G, seq, wg);
+        int most = 0;
+        for (int g = 0; g < G; ++g) most = std::max(most, wg[(size_t)g + 1].pos - wg[(size_t)g].pos);
+        if (sk_cf_busiest(it.T, G) != most) return fail("busiest workgroup", most, sk_cf_busiest(it.T, G));
         for (int g = 0; g <= G; ++g) {
             const int first = sk_cf_first(it.T, G, g);
             if (wg[(size_t)g].pos != first || wg[(size_t)g].iter != first * ST) return fail("workgroup start", g, first);

@@ -208,8 +208,7 @@ SinglePlan sk_single_plan(int M, int NT, int ST, int scale_f32, int sps, int cu_
     if (!sk_wide_supported(scale_f32, sps)) return plan;
     const int Tw = sk_tiles(M, NT, kGemmWideNTW, kGemmFM);
     const int Gw = std::min(sk_max_grid(cu_count), Tw);
-    int busiest = 0;   // tiles of the busiest workgroup in closed-form order
-    for (int g = 0; g < Gw; ++g) busiest = std::max(busiest, sk_cf_first(Tw, Gw, g + 1) - sk_cf_first(Tw, Gw, g));
+    const int busiest = sk_cf_busiest(Tw, Gw);
     const double load = (double)Gw / cu_count;
     const double wide = busiest * (ST * (kStageUs + kStageBusyUs * load) * kGemmWideStageCost + kTileUs);
     if (wide < stream_k) plan = SinglePlan{true, kGemmWideNTW, kGemmFM, Gw, wide, (int64_t)2 * busiest * ST};
@@ -229,8 +228,7 @@ SinglePlan sk_single_plan(int M, int NT, int ST, int scale_f32, int sps, int cu_
 SinglePlan sk_half_plan(int M, int NT, int ST, int cu_count) {
     const int T = sk_tiles(M, NT, kGemmNTW, kGemmHalfFM);
     const int G = std::min(sk_max_grid(cu_count), T);
-    int busiest = 0;
-    for (int g = 0; g < G; ++g) busiest = std::max(busiest, sk_cf_first(T, G, g + 1) - sk_cf_first(T, G, g));
+    const int busiest = sk_cf_busiest(T, G);
     const double load = (double)G / cu_count;
     return SinglePlan{true, kGemmNTW, kGemmHalfFM, G, 2.5 + busiest * (ST * (0.90 + 0.13 * load) + 3.7 + 3.0 * load),
                       (int64_t)busiest * ST};

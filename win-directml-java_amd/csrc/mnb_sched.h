@@ -86,6 +86,16 @@ MNB_HD inline int32_t sk_cf_base(int32_t T, int32_t G, int32_t g) {
     const int32_t X = G % 8 == 0 ? 8 : 1, per = G / X;
     return sk_cf_xcd_start(T, X, g / per) + g % per;
 }
+// Most tiles of any workgroup.
+inline int32_t sk_cf_busiest(int32_t T, int32_t G) {
+    const int32_t X = G % 8 == 0 ? 8 : 1, per = G / X;
+    int32_t most = 0;
+    for (int32_t x = 0; x < X; ++x) {
+        const int32_t n = (sk_cf_xcd_start(T, X, x + 1) - sk_cf_xcd_start(T, X, x) + per - 1) / per;
+        if (n > most) most = n;
+    }
+    return most;
+}
 MNB_HD inline int32_t sk_cf_step(int32_t G) { return G % 8 == 0 ? G / 8 : G; }
 // Tile (m-tile + n-group * MT) at block-order position q of an item with MT
 // m-tiles and NG n-groups: chunks of up to 4 m-tiles, each cut into blocks of
