@@ -298,7 +298,10 @@ def test_quantizer_bytes_where_the_reciprocal_cannot_decide(ctx, rows, cols, bs,
         w.close()
 
 
-@pytest.mark.parametrize("K,bs,offset", [(896, 128, 0), (896, 32, 1), (132, 16, 0), (90, 32, 0), (2052, 128, 0)])
+@pytest.mark.parametrize("K,bs,offset", [(896, 128, 0), (896, 32, 1), (132, 16, 0), (90, 32, 0), (2052, 128, 0),
+                                         # every length of a row's last piece, the shortest rows
+                                         (129, 32, 0), (130, 16, 1), (131, 64, 0), (133, 32, 1), (134, 16, 0), (135, 128, 1),
+                                         (1, 16, 0), (5, 32, 3), (7, 16, 0)])
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 def test_dequantize_into_aligned_and_unaligned_rows(ctx, K, bs, offset, dtype):
     """Rows of out at every alignment the kernel tells apart (16-byte rows,

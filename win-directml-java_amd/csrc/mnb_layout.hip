@@ -10,7 +10,10 @@
 namespace mnb {
 
 typedef u32x4_t u32x4_dq_alias_t __attribute__((may_alias));
-typedef u32x4_t u32x4_row_t __attribute__((may_alias, aligned(2)));   // 16 bytes of a row of fp16 or fp32
+// 16, 8 and 4 bytes of a row of fp16 or fp32
+typedef u32x4_t u32x4_row_t __attribute__((may_alias, aligned(2)));
+typedef u32x2_t u32x2_row_t __attribute__((may_alias, aligned(2)));
+typedef uint32_t u32_row_t __attribute__((may_alias, aligned(2)));
 constexpr int kDequantThreads = 256;
 
 WeightGeom make_geom(int32_t N, int32_t K, int32_t bs) {
@@ -261,6 +264,18 @@ hipError_t launch_stage_x(const void *x, int32_t x_type, int32_t M, int32_t K, i
                              : stage_x_typed((const _Float16 *)x, M, K, ldx, out, stream);
 }
 
+// Stores the first n (fewer than there are) of the fp32 or fp16 values in v.
+__device__ __forceinline__ void store_head(float *p, const u32x4_t &v, int n) {
+    if (n & 2) *(u32x2_row_t *)p = (u32x2_t){v[0], v[1]};
+    if (n & 1) p[n - 1] = __builtin_bit_cast(float, n & 2 ? v[2] : v[0]);
+}
+__device__ __forceinline__ void store_head(_Float16 *p, const u32x4_t &v, int n) {
+    const uint32_t lo = n & 4 ? v[2] : v[0], hi = n & 4 ? v[3] : v[1];
+    if (n & 4) *(u32x2_row_t *)p = (u32x2_t){v[0], v[1]};
+    if (n & 2) *(u32_row_t *)(p + (n & 4)) = lo;
+    if (n & 1) p[n - 1] = __builtin_bit_cast(_Float16, (uint16_t)(n & 2 ? hi : lo));
+}
+
 // w = float(q - zp) * scale, formed as (float(q - zp) * stored scale) *
 // 2^-fold_exp: the power of two makes the two roundings one.
 //
@@ -268,9 +283,16 @@ hipError_t launch_stage_x(const void *x, int32_t x_type, int32_t M, int32_t K, i
 // One wave per tile: its nibbles pass through LDS, so that every store
 // instruction writes whole consecutive pieces of 16 bytes per lane (two rows
 // of 512 bytes in fp32, four of 256 in fp16).  Qwen's [151936, 896] head with
-// fp32 scales to fp32: 100-106 us (618 MB, 5.9 TB/s; 108-112 with cached stores); a thread per 8 k with a
-// load of its own dword and 32-byte strided stores took 332-334 us.  VEC: rows
-// of out are 16-byte aligned; otherwise the same lanes store elements.
+// fp32 scales to fp32: 100-106 us (618 MB, 5.9 TB/s; 108-112 with cached
+// stores); a thread per 8 k with a load of its own dword and 32-byte strided
+// stores took 332-334 us.  VEC: rows of out are 16-byte aligned.  Otherwise the
+// pieces are stored at the alignment they have, cached (lines at the pieces'
+// ends are shared), and a row's shorter last piece in parts of 8, 4 and 2
+// bytes: 3072 -> 9216 off by one element to fp32 25 us, to fp16 17 (a thread per
+// 8 k 71 and 39, element stores 46 and 42, non-temporal 37 and 21); 1001 ->
+// 9728 to fp16 7.3 (17.3; 19.8).  The tile index stays uniform and 32-bit:
+// small matrices are bound by one wave's latency (203 -> 4096 to fp16 4.4 us;
+// 4.8 with a 64-bit division per lane).
 template <typename ScaleT, typename OutT, bool HAS_ZP, bool VEC>
 __global__ __launch_bounds__(kDequantThreads) void dequant_kernel(WeightGeom g, const uint32_t *__restrict__ q_t,
                                                                   const ScaleT *__restrict__ s_t,
@@ -283,20 +305,21 @@ __global__ __launch_bounds__(kDequantThreads) void dequant_kernel(WeightGeom g, 
     // (RPS rows, 4 dwords of each of 4 lane groups) then touch distinct banks
     constexpr int GSTRIDE = 64 + 8;
     __shared__ __align__(16) uint32_t smem[kDequantThreads / 64][4 * GSTRIDE];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t tile = (int64_t)blockIdx.x * (kDequantThreads / 64) + wave;
-    if (tile >= (int64_t)g.NT * g.ST) return;   // whole waves; a wave uses its own LDS only
-    const int nt = (int)(tile / g.ST), st = (int)(tile - (int64_t)nt * g.ST);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t tile = blockIdx.x * (kDequantThreads / 64) + wave;   // below 2^31: a tile is 1 KiB of nibbles
+    if (tile >= (uint32_t)g.NT * (uint32_t)g.ST) return;   // whole waves; a wave uses its own LDS only
+    const int nt = (int)(tile / (uint32_t)g.ST), st = (int)(tile - (uint32_t)nt * (uint32_t)g.ST);
     *(u32x4_dq_alias_t *)&smem[wave][(lane >> 4) * GSTRIDE + (lane & 15) * 4] =
         gld_nt((const u32x4_t *)q_t + (size_t)tile * 64 + lane);
     asm volatile("" ::: "memory");   // a wave's LDS accesses run in order
     const int kk = (lane % LPR) * E;            // k of the lane's elements inside the tile
     const int k0 = st * kTileK + kk;
     const int j = kk / 32, gg = (kk % 32) / 8, i0 = kk % 8;
-    const int si = g.bs >= kTileK ? 0 : kk / g.bs;
+    const int si = kk * g.SPS / kTileK;   // the block of kk; 0 where a block spans the tile
     const float unfold = pow2f(-g.fold_exp);
     float sc[kTileRows / RPS];
     int zv[kTileRows / RPS];
+    u32x4_t ov[kTileRows / RPS];
 #pragma unroll
     for (int i = 0; i < kTileRows / RPS; ++i) {
         const size_t e = (size_t)tile * kTileRows + i * RPS + lane / LPR;
@@ -319,14 +342,22 @@ __global__ __launch_bounds__(kDequantThreads) void dequant_kernel(WeightGeom g, 
             o[x] = (OutT)v;
         }
         OutT *p = out + (size_t)n * g.K + k0;
+        __builtin_memcpy(&ov[i], o, 16);
         if constexpr (VEC) {
-            u32x4_t ov;
-            __builtin_memcpy(&ov, o, 16);
-            if (n < g.N && k0 < g.K) __builtin_nontemporal_store(ov, (u32x4_t *)p);
+            if (n < g.N && k0 < g.K) __builtin_nontemporal_store(ov[i], (u32x4_t *)p);
         } else {
+            if (n < g.N && k0 + E <= g.K) *(__attribute__((address_space(1))) u32x4_row_t *)p = ov[i];
+        }
+    }
+    if constexpr (!VEC) {
+        // the last, shorter piece of the rows
+        const int rem = g.K - k0;
+        if (rem > 0 && rem < E) {
 #pragma unroll
-            for (int x = 0; x < E; ++x)
-                if (n < g.N && k0 + x < g.K) p[x] = o[x];
+            for (int i = 0; i < kTileRows / RPS; ++i) {
+                const int n = nt * kTileRows + i * RPS + lane / LPR;
+                if (n < g.N) store_head(out + (size_t)n * g.K + k0, ov[i], rem);
+            }
         }
     }
 }
