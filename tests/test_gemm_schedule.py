@@ -293,7 +293,6 @@ def test_k_sliced_blocks_are_the_fastest_measured(checker):
         ((128, 8192, 3072), (2, 4)),    # 32x64 19.12
         ((137, 4096, 9850), (4, 4)),    # 64x64 34.56; 32x64 41.92
         ((78, 8192, 7050), (4, 4)),     # 64x64 27.86; 32x64 34.70
-        ((129, 13938, 3133), (2, 4)),   # 32x64 34.8; 48x64 36.7 (bs 128)
         ((231, 512, 1760), (2, 2)),     # 32x32 4.72; 32x64 5.12 (K = 512: the first model)
         ((80, 512, 6023), (2, 2)),      # 32x32 5.62; 64x64 7.49 (K = 512: the first model)
     ]

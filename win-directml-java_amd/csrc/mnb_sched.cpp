@@ -296,10 +296,7 @@ int ks_waves(int ST) { return ST < kKsMaxWaves ? ST : kKsMaxWaves; }
 // short tiles).  On shorter K, where several workgroups share a CU, it
 // misjudged the blocks, so those keep the first model.  (The 64 x 64 block's
 // r2 and thr2 are those of its one-round reduction: 3.6 and 470 against 4.603
-// and 422.6 with the reduction in rounds.  The 32 x 64 block's rate rose with
-// it too, by 5-8%; 715 against 693.6 takes the half of that which keeps the
-// two blocks' order right: 13938 -> 3133 at M = 129 takes 34.8 us with 32 x 64
-// blocks, 36.7 with 48 x 64 ones.)
+// and 422.6 with the reduction in rounds.)
 struct KsCost {
     int mb, ntw;
     double c, k, thr;
@@ -308,7 +305,7 @@ struct KsCost {
 static const KsCost kKsCosts[] = {
     {2, 1, 3.06, 0.88, 2114.0, 2.417, 0.878, 0.687, 2223.1},
     {2, 2, 2.92, 1.16, 1138.0, 1.346, 1.311, 1.715, 1376.7},
-    {2, 4, 3.86, 1.58, 757.0, 1.177, 1.754, 2.901, 715.0},
+    {2, 4, 3.86, 1.58, 757.0, 1.177, 1.754, 2.901, 693.6},
     {4, 4, 5.50, 2.30, 469.0, 0.932, 2.543, 3.6, 470.0},
 };
 constexpr int kKsRoundCostMinST = 6;
