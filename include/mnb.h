@@ -211,11 +211,12 @@ int32_t mnb_matmul(mnb_context *ctx, const mnb_weight *w, int32_t M, const void 
  * run (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc).  Same arguments, checks, kernels and results as mnb_matmul
  * without MNB_HOST_MEMORY (which it refuses).  The GEMM's split-tile partial
- * sums and the fp16 copy of x (made when x is fp32, not 16-byte aligned or K
- * is not a multiple of 8) live in a fixed 80 MiB device array of the library
+ * sums and the fp16 copy of x (made when x is not 16-byte aligned, K is not a
+ * multiple of 8, or x is fp32 and not read in place, as some products of at
+ * most 16 rows do) live in a fixed 80 MiB device array of the library
  * instead of context buffers: 64 MiB of partial tiles and at most 16 MiB of
- * staged x, M * roundup(K, 8) * 2 bytes (a larger staging need fails with
- * MNB_ERR_INVALID_ARGUMENT).  Each GPU holds its own array for the life of
+ * staged x, M * roundup(K, 8) * 2 bytes (more than that, for any fp32,
+ * unaligned or K % 8 != 0 x, fails with MNB_ERR_INVALID_ARGUMENT).  Each GPU holds its own array for the life of
  * the process; every call on one GPU shares it, so calls that overlap on one
  * GPU (concurrent streams, other threads) race: order them. */
 int32_t mnb_matmul_noalloc(mnb_context *ctx, const mnb_weight *w, int32_t M, const void *x, int32_t x_type,

@@ -237,11 +237,10 @@ __global__ __launch_bounds__(64 * kKsMaxWaves) void gemm_ks_kernel(KsParams p) {
     // another (same box, block forced, us): 64 x 64 3072 -> 3072 at M = 64 13.2
     // -> 11.6, 896 -> 9728 8.3 -> 7.2, 3072 -> 9216 at M = 200 40.4 -> 35.0;
     // 32 x 64 3072 -> 3072 at M = 64 9.2 -> 8.6; 32 x 32 7.2 -> 7.0, 3072 -> 9216
-    // at M = 200 45.2 -> 41.2; 32 x 16 8.8 -> 8.7 (3% slower where it runs
-    // many rounds, which it is not chosen for).  Loading as many units as the
-    // largest workgroup has waves, whatever W is, cost short K up to a
-    // quarter (32 x 64, 128 -> 4096 4.6 -> 5.8, 256 -> 4096 4.4 -> 5.0); one wave
-    // alone stores its block as it is (4.1).
+    // at M = 200 45.2 -> 41.2; 32 x 16 8.8 -> 8.7 (864 -> 20461 at M = 20 10.4 ->
+    // 10.6).  Loading as many units as the largest workgroup has waves,
+    // whatever W is, cost short K up to a quarter (32 x 64, 128 -> 4096 4.6 ->
+    // 5.8, 256 -> 4096 4.4 -> 5.0); one wave alone stores its block as it is (4.1).
     if (W == 1) {
 #pragma unroll
         for (int q = 0; q < U; ++q) store_unit(q, acc[q / NTW][q % NTW]);

@@ -269,7 +269,7 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_tiles_kernel(WeightGeo
 
 // Multiplies the quantized scales by 2^fold_exp, the weight's fold exponent
 // from the quantizer's n_part partial maxima (every workgroup reduces them,
-// at most 8 KiB, for itself), and stores the exponent in *fold.
+// at most 4 KiB, for itself), and stores the exponent in *fold.
 __global__ __launch_bounds__(kQuantThreads) void fold_scales_kernel(float4_t *__restrict__ s, size_t n4,
                                                                     const float *__restrict__ part, int n_part,
                                                                     int32_t *__restrict__ fold) {
